@@ -72,3 +72,69 @@ def test_non_finite_operands(lib, ta, tb, beta):
     assert torch.equal(torch.isinf(got), inf) and torch.equal(got[inf], want[inf])
     fin = torch.isfinite(want)
     np.testing.assert_allclose(got[fin].numpy(), want[fin].numpy(), rtol=2e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(150, 70, 515), (300, 260, 31), (64, 33, 16)])
+def test_blocks_taken_again(lib, M, N, K, ta, tb):
+    """Infinities in the last row, the last column and the last k (K with and without a remainder
+    of 16), in batches that take every tile shape: the outputs beside them stay those of the fp32
+    sum."""
+    for batch in (1, 24):
+        g = torch.Generator().manual_seed(M + batch)
+        A = torch.randn((batch, M, K), generator=g)
+        B = torch.randn((batch, K, N), generator=g)
+        A[:, M - 1, K - 1] = float("inf")
+        A[:, 3, 0] = float("-inf")
+        B[:, K // 2, N - 1] = float("inf")
+        # dense sums without the infinite terms; those rows and columns by their signs
+        A0, B0 = A.clone(), B.clone()
+        A0[torch.isinf(A0)] = 0.0
+        B0[torch.isinf(B0)] = 0.0
+        want, mag = product64(A0, B0, False, False)
+        want[:, M - 1] = float("inf") * B[:, K - 1].sign().double()
+        want[:, 3] = float("-inf") * B[:, 0].sign().double()
+        col = want[:, :, N - 1]
+        add = float("inf") * A[:, :, K // 2].sign().double()
+        want[:, :, N - 1] = torch.where(torch.isinf(col), col + add, add)
+        dev = lambda x, t: (x.transpose(1, 2) if t else x).contiguous().cuda()
+        C = torch.empty((batch, M, N), device="cuda:0")
+        run(lib, dev(A, ta), dev(B, tb), C, M, N, K, ta, tb)
+        got = C.cpu().double()
+        fin = torch.isfinite(want)
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+        # a rounding of 2^-23 of the magnitudes so far per k, whichever form a block takes
+        lim = (K + 8) * 2.0 ** -23 * mag
+        assert bool(((got - want).abs()[fin] <= lim[fin]).all())
+
+
+def test_infinity_cost(lib):
+    """An infinity in a row and in a column must not cost many times the product: their outputs are
+    taken again by whole waves (2.9 times the product at 128 x 128 x 32768; a lane's serial sums of
+    32768 terms took 77 times)."""
+    M, N, K = 128, 128, 32768
+    g = torch.Generator(device="cuda:0").manual_seed(1)
+    A = torch.randn((1, M, K), generator=g, device="cuda:0")
+    B = torch.randn((1, N, K), generator=g, device="cuda:0")
+    C = torch.empty((1, M, N), device="cuda:0")
+
+    def time_us():
+        run(lib, A, B, C, M, N, K, False, True)
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = float("inf")
+        for _ in range(5):
+            e[0].record()
+            lib.matmul_batched_strided(A, B, C, M, N, K, M * K, K * N, M * N, 1, False, True, 1.0,
+                                       0.0)
+            e[1].record()
+            torch.cuda.synchronize()
+            best = min(best, e[0].elapsed_time(e[1]) * 1e3)
+        return best
+
+    plain = time_us()
+    A[0, 7, 11] = B[0, 9, 12] = float("inf")
+    again = time_us()
+    print(f"{plain:.0f} us, with infinities {again:.0f} us")
+    assert not bool(torch.isfinite(C[0, 7]).any()) and not bool(torch.isfinite(C[0, :, 9]).any())
+    assert again < 8 * plain
