@@ -138,3 +138,44 @@ def test_infinity_cost(lib):
     print(f"{plain:.0f} us, with infinities {again:.0f} us")
     assert not bool(torch.isfinite(C[0, 7]).any()) and not bool(torch.isfinite(C[0, :, 9]).any())
     assert again < 8 * plain
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("up,down", [(100, -125), (100, -115), (90, -100), (60, -60), (102, -102)])
+def test_scaled_operands(lib, up, down, ta, tb):
+    """Operands scaled by powers of two, which round nothing: the same bits as without, down to the
+    smallest normal numbers and up to 2^103."""
+    M, N, K = 70, 130, 100
+    g = torch.Generator().manual_seed(2)
+    draw = lambda *n: (1.0 + torch.rand(n, generator=g)) * (torch.randint(0, 2, n, generator=g) * 2 - 1)
+    A, B = draw(1, M, K).cuda(), draw(1, K, N).cuda()
+    dev = lambda x, t: (x.transpose(1, 2) if t else x).contiguous()
+    C = [torch.empty((1, M, N), device="cuda:0") for _ in range(3)]
+    run(lib, dev(A, ta), dev(B, tb), C[0], M, N, K, ta, tb)
+    run(lib, dev(A * 2.0 ** up, ta), dev(B * 2.0 ** down, tb), C[1], M, N, K, ta, tb)
+    run(lib, dev(A * 2.0 ** down, ta), dev(B * 2.0 ** up, tb), C[2], M, N, K, ta, tb)
+    want = C[0] * 2.0 ** (up + down)
+    assert torch.equal(C[1], want) and torch.equal(C[2], want)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+@pytest.mark.parametrize("sa,sb", [
+    (-149, 120), (-140, 126), (-135, 0), (-74, -73), (-126, -20),  # subnormal operands, results
+    (104, -100), (126, -126), (120, 1), (45, 45), (63, 58)])       # beyond the planes' range
+def test_operand_range(lib, sa, sb, ta, tb):
+    """The ends of fp32's range, in operands and results."""
+    M, N, K = 70, 66, 40
+    g = torch.Generator().manual_seed(3)
+    A = torch.ldexp(torch.rand((1, M, K), generator=g, dtype=torch.float64) + 0.5,
+                    torch.tensor(sa)).float().double()
+    B = torch.ldexp(torch.randn((1, K, N), generator=g, dtype=torch.float64) * 0.125,
+                    torch.tensor(sb)).float().double()
+    want, mag = product64(A, B, False, False)
+    assert bool((mag < 2.0 ** 128).all())
+    dev = lambda x, t: (x.transpose(1, 2) if t else x).contiguous().float().cuda()
+    C = torch.empty((1, M, N), device="cuda:0")
+    run(lib, dev(A, ta), dev(B, tb), C, M, N, K, ta, tb)
+    # 2^-23 of the magnitudes so far for each of K roundings at most, and a subnormal result's last
+    # bit for each
+    lim = (K + 8) * (2.0 ** -23 * mag + 2.0 ** -149)
+    assert bool(((C.cpu().double() - want).abs() <= lim).all())
