@@ -179,3 +179,21 @@ def test_operand_range(lib, sa, sb, ta, tb):
     # bit for each
     lim = (K + 8) * (2.0 ** -23 * mag + 2.0 ** -149)
     assert bool(((C.cpu().double() - want).abs() <= lim).all())
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,batch", [(1, 1, 1), (65, 130, 2), (300, 257, 30)])
+def test_short_products(lib, M, N, batch, ta, tb):
+    """One k: the rounded product itself; two and three: one rounding for each."""
+    g = torch.Generator(device="cuda:0").manual_seed(4)
+    for K in (1, 2, 3):
+        A = torch.randn((batch, M, K), generator=g, device="cuda:0")
+        B = torch.randn((batch, K, N), generator=g, device="cuda:0")
+        dev = lambda x, t: (x.transpose(1, 2) if t else x).contiguous()
+        for alpha, beta in ((1.0, 0.0), (1.0, 1.0)):
+            C = torch.zeros((batch, M, N), device="cuda:0")
+            run(lib, dev(A, ta), dev(B, tb), C, M, N, K, ta, tb, alpha, beta)
+            want, mag = product64(A, B, False, False)
+            if K == 1:
+                assert torch.equal(C, A * B)
+            assert bool(((C.double() - want).abs() <= K * 2.0 ** -24 * mag + 2.0 ** -149).all())
