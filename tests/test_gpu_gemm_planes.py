@@ -197,3 +197,14 @@ def test_short_products(lib, M, N, batch, ta, tb):
             if K == 1:
                 assert torch.equal(C, A * B)
             assert bool(((C.double() - want).abs() <= K * 2.0 ** -24 * mag + 2.0 ** -149).all())
+
+
+def test_more_tiles_than_one_launch_holds(lib):
+    """9 437 184 products of 1 x 68 x 4: 2^24 and more 64 x 64 tiles."""
+    n, N, K = 9 * 2 ** 20, 68, 4
+    A = torch.arange(1.0, 5.0, device="cuda:0")
+    B = torch.arange(float(K * N), device="cuda:0")
+    C = torch.zeros(n * N, device="cuda:0")
+    lib.matmul_batched_strided(A, B, C, 1, N, K, 0, 0, N, n, False, False, 1.0, 0.0)
+    want = (A.cpu() @ B.cpu().view(K, N)).cuda()
+    assert bool((C.view(n, N) == want).all())

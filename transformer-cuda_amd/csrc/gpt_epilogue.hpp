@@ -173,7 +173,7 @@ template <bool TA, bool TB, class Map>
 void product_map(int M, int N, int K, const float* A, const float* B, const Map& map,
                  bool aligned, float* scratch, hipStream_t s) {
     const Plan p = plan(M, N, K, Map::kArrays);
-    const Problem g{A, B, M, N, K, 0, 0, kGemmFull, p.kslice, 0, 0, 0};
+    const Problem g{A, B, M, N, K, 0, 0, kGemmFull, p.kslice, 0, 0, 0, 0};
     const EpiMap<Map> epi{map, N % 2 == 0 && aligned};
     if (p.slices == 1) {
         launch_tile<TA, TB>(p.tile, g, 1, epi, s);
@@ -196,7 +196,7 @@ template <bool TA, bool TB>
 void product_plain(int M, int N, int K, const float* A, const float* B, float* C, float* scratch,
                    hipStream_t s) {
     const Plan p = plan(M, N, K);
-    const Problem g{A, B, M, N, K, 0, 0, kGemmFull, p.kslice, 0, 0, 0};
+    const Problem g{A, B, M, N, K, 0, 0, kGemmFull, p.kslice, 0, 0, 0, 0};
     const long long mn = static_cast<long long>(M) * N;
     launch_tile<TA, TB>(p.tile, g, p.slices, plain(p.slices > 1 ? scratch : C, N, mn), s);
     if (p.slices > 1) sum_slices(scratch, p.slices, mn, C, s);
