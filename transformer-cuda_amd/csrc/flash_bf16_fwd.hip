@@ -34,6 +34,7 @@
 // fp32 and split in registers (its planes written out for the backward); P is split into
 // planes as it leaves the softmax.  The tiles are 32 keys deep, so that the double-buffered
 // planes (55 KB at d = 64) leave room for two workgroups per CU.
+#include <float.h>
 #include <math.h>
 
 #include <type_traits>
@@ -170,13 +171,15 @@ __device__ __forceinline__ void softmax_step(f32x16& s, SubState<D>& st, bf16x8 
     st.m_true = fmaxf(st.m_true, mx);
     if (__builtin_amdgcn_ballot_w64((mx - st.m_used) * c > kRescaleLog2) != 0) {
         const float m_new = fmaxf(st.m_used, mx);
-        const float alpha = exp2_fast((st.m_used - m_new) * c);  // 0 at the start
+        const float alpha = exp2_fast((st.m_used - fmaxf(m_new, -FLT_MAX)) * c);  // 0 at the start
         st.l *= alpha;
 #pragma unroll
         for (int dt = 0; dt < D / 32; ++dt) st.acc[dt] *= alpha;
         st.m_used = m_new;
     }
-    const float mc = st.m_used * c;
+    // finite references (here and above): keys with scores of -inf weigh nothing where the wave has
+    // met no others yet
+    const float mc = fmaxf(st.m_used * c, -FLT_MAX);
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = exp2_fast(fmaf(s[r], c, -mc));
     st.l += xhalf_sum(sum_tree16(s));

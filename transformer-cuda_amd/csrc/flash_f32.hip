@@ -45,6 +45,7 @@
 // kernel's sums), the dK/dV kernel writing dS as well (its DS form), then dQ = scale * dS K
 // from the stored dS (flash_bwd_dq_ds_f32_kernel), which leaves out the dQ kernel's second
 // computation of S and dP.
+#include <float.h>
 #include <math.h>
 
 #include <type_traits>
@@ -378,8 +379,10 @@ __device__ __forceinline__ void fwd_chunk(const float* __restrict__ kh,
         for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
         mx = xhalf_max(mx);
         const float m_new = fmaxf(m_raw, mx);
-        const float alpha = exp2_fast((m_raw - m_new) * c);  // 0 on the first tile
-        const float mc = m_new * c;
+        // 0 on the first tile; finite references, so that keys with scores of -inf weigh nothing
+        // where the wave has met no others yet
+        const float alpha = exp2_fast((m_raw - fmaxf(m_new, -FLT_MAX)) * c);
+        const float mc = fmaxf(m_new * c, -FLT_MAX);
         float rs = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -594,8 +597,10 @@ __global__ __launch_bounds__(kWave* kFwdSharedWaves) void flash_fwd_f32_shared_k
         for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
         mx = xhalf_max(mx);
         const float m_new = fmaxf(m_raw, mx);
-        const float alpha = exp2_fast((m_raw - m_new) * c);  // 0 on the first tile
-        const float mc = m_new * c;
+        // 0 on the first tile; finite references, so that keys with scores of -inf weigh nothing
+        // where the wave has met no others yet
+        const float alpha = exp2_fast((m_raw - fmaxf(m_new, -FLT_MAX)) * c);
+        const float mc = fmaxf(m_new * c, -FLT_MAX);
         float rs = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
