@@ -52,6 +52,7 @@
 
 #include "bf16_tile.hpp"
 #include "device_common.hpp"
+#include "forms.hpp"
 #include "launch.hpp"
 #include "lds_dma.hpp"
 #include "sched.hpp"
@@ -1427,39 +1428,11 @@ QueueSlot* launch_slot(Family f, std::atomic<unsigned>& ticket, hipStream_t stre
     return base + next_queue_slot(ticket);
 }
 
-// A stage on shared tiles (flash_*_f32_shared_kernel, 128 rows per workgroup) where it is the
-// faster one, else the persistent per-wave kernel, whose four waves share out every task's tile
-// range.  A workgroup of the shared form walks the whole range of its rows by itself, so it needs
-// two of them on every CU and an even last round; with fewer, its time is that of the longest
-// range.  Measured (one process, us, shared -> per-wave: forward, dQ, dK/dV), d = 64:
-//   B*H 8, T 1024 (64 workgroups)     78 -> 25    116 -> 63    150 -> 47
-//   B*H 27, T 777 (189)               63 -> 39     91 -> 75    123 -> 73
-//   B*H 64, T 512 (256)               42 -> 30     63 -> 53     80 -> 61
-//   B*H 48, T 1024 (384: 1.5 a CU)   100 -> 69    149 -> 128   191 -> 141
-//   B*H 96, T 777 (672, 12% empty)    96 -> 85    146 -> 129   179 -> 169
-//   B*H 64, T 1024 (512)              90 -> 88    133 -> 146   168 -> 177
-//   B*H 96, T 1024 (768)             127 -> 130   194 -> 193   253 -> 251
-// and beyond T = 2048 its static block order balances the causal ranges worse than the queue
-// (B1 H12 T8192 forward 886 per-wave, 1086 shared).  d = 128:
-//   B*H 16, T 2048 (256)             277 -> 182   416 -> 322   568 -> 364
-//   B*H 48, T 777 (336)              140 -> 107   165 -> 151   231 -> 210
-//   B*H 27, T 2048 (432)             373 -> 309   425 -> 413   582 -> 624
-//   B*H 64, T 1024 (512)             160 -> 204   248 -> 263   340 -> 409
-// d = 32: B8 H12 T1024 forward 72 per-wave, 74 shared.
-bool on_shared_tiles(Family f, int D, int T, int BH) {
-    if (D == 32) return false;
-    const long long nblk = static_cast<long long>(BH) * ((T + 127) / 128);
-    if (D == 128) return nblk >= (f == Family::Dkdv ? 352 : 512);
-    if (T > 2048 || nblk < 512) return false;
-    const double rounds = static_cast<double>((nblk + 255) / 256);
-    return nblk >= 1024 || static_cast<double>(BH) * T / 128.0 >= 0.9 * 256.0 * rounds;
-}
-
 template <int D>
 void fwd_dispatch(const float* q, const float* k, const float* v, float* o, float* m_out,
                   float* l_out, int BH, int T, float scale, const HeadView& xv,
                   const HeadView& ov, hipStream_t stream) {
-    if (on_shared_tiles(Family::Fwd, D, T, BH)) {
+    if (on_shared_tiles(Stage::Fwd, D, T, BH)) {
         constexpr int kBlock = kTile * kFwdSharedWaves;
         const int nblk = (T + kBlock - 1) / kBlock;
         const auto kernel = flash_fwd_f32_shared_kernel<D>;
@@ -1484,7 +1457,7 @@ void dq_dispatch(const float* q, const float* k, const float* v, const float* o,
                  const float* dO, const float* m, const float* l, float* dq, float* Dws, int BH,
                  int T, float scale, const HeadView& xv, const HeadView& ov, const HeadView& gv,
                  hipStream_t stream) {
-    if (on_shared_tiles(Family::Dq, D, T, BH)) {
+    if (on_shared_tiles(Stage::Dq, D, T, BH)) {
         constexpr int kBlock = kTile * kFwdSharedWaves;
         const int nblk = (T + kBlock - 1) / kBlock;
         const auto kernel = flash_bwd_dq_f32_shared_kernel<D>;
@@ -1510,7 +1483,7 @@ void dkdv_launch(const float* q, const float* k, const float* v, const float* dO
                  const float* m, const float* l, const float* Dws, float* dk, float* dv, int BH,
                  int T, float scale, const HeadView& xv, const HeadView& ov, const HeadView& gv,
                  float* ds, hipStream_t stream) {
-    if (on_shared_tiles(Family::Dkdv, D, T, BH)) {
+    if (on_shared_tiles(Stage::Dkdv, D, T, BH)) {
         constexpr int kBlock = kTile * kFwdSharedWaves;
         const int nblk = (T + kBlock - 1) / kBlock;
         const auto kernel = flash_bwd_dkdv_f32_shared_kernel<D, DS>;

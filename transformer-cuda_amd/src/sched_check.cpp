@@ -10,15 +10,21 @@
 //     (non-increasing causal work) within a head, and a group's blocks all come before the
 //     next group's.
 // And head_group at the bench shapes, with the resident capacities the occupancy query
-// reports for those kernels on MI355X.  Prints "sched_check: all passed" on success.
+// reports for those kernels on MI355X; and the forms that on_shared_tiles picks at shapes where one
+// form measured clearly faster.  Prints "sched_check: all passed" on success.
+//
+// sched_check form STAGE D T BH prints the fp32 form of a call instead (STAGE: fwd, dq, dkdv).
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "bf16_tile.hpp"
+#include "forms.hpp"
 #include "sched.hpp"
 
 using tcamd::head_group;
+using tcamd::Stage;
 using tcamd::bf16t::map_block;
 using tcamd::bf16t::map_block_grouped;
 
@@ -76,7 +82,103 @@ static void check_order(int BH, int nb, bool descending, int order, int G) {
               BH, nb, order, G, i / nb, i % nb, seen[i]);
 }
 
-int main() {
+// fp32 shapes where one form is the faster one by 8% and more: us on shared tiles and per-wave.
+static void check_f32_forms() {
+    const struct {
+        Stage stage;
+        int D, T, BH;
+        double shared, per_wave;
+    } measured[] = {
+        {Stage::Fwd, 64, 100, 64, 13, 7},
+        {Stage::Fwd, 64, 100, 200, 13, 16},
+        {Stage::Fwd, 64, 128, 256, 14, 16},
+        {Stage::Fwd, 64, 230, 256, 31, 38},
+        {Stage::Fwd, 64, 777, 27, 61, 37},
+        {Stage::Fwd, 64, 1024, 8, 78, 23},
+        {Stage::Fwd, 64, 2048, 16, 152, 91},
+        {Stage::Fwd, 64, 512, 256, 83, 105},
+        {Stage::Fwd, 128, 64, 144, 13, 20},
+        {Stage::Fwd, 128, 100, 64, 21, 12},
+        {Stage::Fwd, 128, 100, 200, 23, 37},
+        {Stage::Fwd, 128, 128, 256, 25, 41},
+        {Stage::Fwd, 128, 777, 27, 108, 67},
+        {Stage::Fwd, 128, 1024, 8, 139, 43},
+        {Stage::Fwd, 128, 2048, 16, 273, 179},
+        {Stage::Fwd, 128, 512, 256, 183, 269},
+        {Stage::Dq, 64, 100, 64, 19, 12},
+        {Stage::Dq, 64, 230, 256, 47, 51},
+        {Stage::Dq, 64, 777, 27, 89, 73},
+        {Stage::Dq, 64, 1024, 8, 115, 61},
+        {Stage::Dq, 64, 2048, 16, 226, 180},
+        {Stage::Dq, 128, 100, 64, 33, 20},
+        {Stage::Dq, 128, 100, 200, 35, 38},
+        {Stage::Dq, 128, 128, 256, 38, 42},
+        {Stage::Dq, 128, 777, 27, 162, 122},
+        {Stage::Dq, 128, 1024, 8, 210, 108},
+        {Stage::Dq, 128, 1200, 96, 572, 525},
+        {Stage::Dq, 128, 2048, 16, 414, 321},
+        {Stage::Dkdv, 64, 100, 64, 23, 12},
+        {Stage::Dkdv, 64, 100, 200, 24, 27},
+        {Stage::Dkdv, 64, 230, 256, 58, 70},
+        {Stage::Dkdv, 64, 777, 27, 123, 71},
+        {Stage::Dkdv, 64, 600, 144, 143, 155},
+        {Stage::Dkdv, 64, 1024, 8, 150, 45},
+        {Stage::Dkdv, 64, 2048, 16, 294, 182},
+        {Stage::Dkdv, 64, 512, 256, 179, 200},
+        {Stage::Dkdv, 128, 64, 144, 24, 36},
+        {Stage::Dkdv, 128, 100, 64, 43, 21},
+        {Stage::Dkdv, 128, 100, 200, 46, 66},
+        {Stage::Dkdv, 128, 128, 256, 50, 78},
+        {Stage::Dkdv, 128, 777, 27, 230, 136},
+        {Stage::Dkdv, 128, 1024, 8, 285, 85},
+        {Stage::Dkdv, 128, 2048, 16, 563, 365},
+        {Stage::Dkdv, 128, 512, 256, 412, 526},
+        // the whole dS-first backward
+        {Stage::Dkdv, 64, 64, 144, 24, 30},
+        {Stage::Dkdv, 64, 100, 64, 37, 25},
+        {Stage::Dkdv, 64, 100, 200, 41, 50},
+        {Stage::Dkdv, 64, 128, 256, 44, 56},
+        {Stage::Dkdv, 64, 230, 256, 89, 127},
+        {Stage::Dkdv, 64, 777, 27, 174, 119},
+        {Stage::Dkdv, 64, 600, 144, 215, 273},
+        {Stage::Dkdv, 64, 1024, 8, 212, 104},
+        {Stage::Dkdv, 64, 1200, 96, 490, 588},
+        {Stage::Dkdv, 64, 2048, 16, 415, 305},
+        {Stage::Dkdv, 64, 512, 256, 283, 365},
+        {Stage::Dkdv, 128, 64, 144, 41, 53},
+        {Stage::Dkdv, 128, 100, 64, 64, 41},
+        {Stage::Dkdv, 128, 100, 200, 70, 91},
+        {Stage::Dkdv, 128, 128, 256, 75, 104},
+        {Stage::Dkdv, 128, 777, 27, 310, 218},
+        {Stage::Dkdv, 128, 1024, 8, 383, 182},
+        {Stage::Dkdv, 128, 2048, 16, 757, 562},
+        {Stage::Dkdv, 128, 512, 256, 580, 700},
+    };
+    for (const auto& m : measured)
+        CHECK(tcamd::on_shared_tiles(m.stage, m.D, m.T, m.BH) == (m.shared < m.per_wave),
+              "stage %d d %d T %d B*H %d takes the slower form (%.0f us shared, %.0f per-wave)",
+              static_cast<int>(m.stage), m.D, m.T, m.BH, m.shared, m.per_wave);
+    // the sizes at which the entry points stop, and B*H * workgroups beyond 2^31
+    for (int st = 0; st < 3; ++st)
+        for (int D : {32, 64, 128})
+            for (int T : {1, 31, 33, 128, 129, 2048, 2049, 1 << 20, 2147483647})
+                for (int BH : {1, 7, 65535}) (void)tcamd::on_shared_tiles(static_cast<Stage>(st), D, T, BH);
+}
+
+static int print_form(char** a) {
+    const char* names[] = {"fwd", "dq", "dkdv"};
+    for (int st = 0; st < 3; ++st)
+        if (std::strcmp(a[0], names[st]) == 0) {
+            const bool shared = tcamd::on_shared_tiles(static_cast<Stage>(st), std::atoi(a[1]),
+                                                       std::atoi(a[2]), std::atoi(a[3]));
+            std::printf("%s\n", shared ? "shared" : "per-wave");
+            return 0;
+        }
+    return 2;
+}
+
+int main(int argc, char** argv) {
+    if (argc == 6 && std::strcmp(argv[1], "form") == 0) return print_form(argv + 2);
     const int bhs[] = {1, 3, 8, 12, 16, 24, 64, 96, 128, 256, 384};
     const int nbs[] = {1, 2, 7, 8, 16, 33, 64};
     for (int BH : bhs)
@@ -104,6 +206,8 @@ int main() {
     CHECK(head_group(100, 64, 512) == 0, "BH 100: %d", head_group(100, 64, 512));
     // G stays below the heads per XCD (G = hpx is the plain order).
     CHECK(head_group(64, 64, 256) == 0, "BH 64: %d", head_group(64, 64, 256));
+
+    check_f32_forms();
 
     if (failures) {
         std::printf("sched_check: %d failures\n", failures);
