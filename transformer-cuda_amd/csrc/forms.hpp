@@ -31,7 +31,7 @@ double makespan(Cost cost, int n, double sum, int heads, bool paired) {
 // a quarter of them and a merge's worth for the other; `merge`, the price of a step of it and the
 // shared form's start are fitted to some 710 shapes of each d, from B*H 1 to 400 and T 33 to 2048,
 // measured in both forms.  The times over all of them are within 0.6% of the better forms'.  Of the
-// slower picks, the forward and dQ have 6 to 11 of more than 5%, of 19% at most.  dK/dV
+// slower picks, the forward and dQ have 4 to 11 of more than 5%, of 19% at most.  dK/dV
 // goes by one rule with and without dS, whose dK and dV are the same bits: as writing dS costs the
 // per-wave form more, the rule leaves it earlier than dK/dV alone would.
 // Measured (us, shared -> per-wave):
@@ -60,8 +60,11 @@ inline bool on_shared_tiles(Stage stage, int D, int T, int BH) {
     const auto wave = [&](int r) { return (nt - r + 3) / 4 + f.merge; };
     const double q = nt / 4, rest = nt % 4;
     const double wave_sum = 2.0 * q * (q + 1.0) + rest * (q + 1.0) + f.merge * nt;
-    // whole rounds in heaviest-first order give every CU the same mix of long and short ones
+    // two workgroups a CU, all resident and nearly full, in serpentine order: each CU has a long and
+    // a short one (B*H 64 T 1024 d 64 dQ 130 shared, 146 per-wave); other whole rounds in
+    // heaviest-first order give every CU about the same mix too
     const long long nblk = static_cast<long long>(nb) * BH;
+    if (nblk == 512 && static_cast<long long>(T) * BH >= 512 * 128 * 85 / 100) return true;
     const bool paired = nblk >= 512 && nblk % 256 == 0;
     return f.start + makespan(shared, nb, shared_sum, BH, paired) <
            f.step * makespan(wave, nt, wave_sum, BH, false);

@@ -133,6 +133,9 @@ static void check_f32_forms() {
         {Stage::Dkdv, 128, 1024, 8, 285, 85},
         {Stage::Dkdv, 128, 2048, 16, 563, 365},
         {Stage::Dkdv, 128, 512, 256, 412, 526},
+        {Stage::Dq, 64, 1024, 64, 130, 146},
+        {Stage::Dq, 64, 2048, 32, 240, 276},
+        {Stage::Dq, 128, 129, 256, 72, 55},
         // the whole dS-first backward
         {Stage::Dkdv, 64, 64, 144, 24, 30},
         {Stage::Dkdv, 64, 100, 64, 37, 25},
