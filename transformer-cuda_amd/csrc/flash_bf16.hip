@@ -52,6 +52,7 @@
 #include <utility>
 
 #include "bf16_tile.hpp"
+#include "forms.hpp"
 #include "device_common.hpp"
 #include "launch.hpp"
 #include "sched.hpp"
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_bf16_kernel(DqArgs
 
 // Stage 1 for few heads: the waves of a workgroup share out the keys of one 32-query block
 // through K and V tiles of their own, and their partial dQ meet in LDS, in wave order (as the
-// forward's flash_fwd_split_kernel; where it runs: split_rows).
+// forward's flash_fwd_split_kernel; where it runs: on_split_rows).
 template <int D, int NP>
 __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_split_kernel(DqArgs<NP> a, int nblk) {
     using S = Swz<D, 32>;
@@ -669,7 +670,7 @@ struct DkdvArgs {
 // Stage 2 for few heads: the waves of a workgroup share out the queries of one 32-key block
 // through Q and dO tiles and statistics of their own, from the last tile down (kDesc's order, which
 // keeps three planes' sums accurate; bf16 takes it too), and their partial dK and dV meet in LDS,
-// in wave order.  Every dS tile is still written by one wave.  Where it runs: split_rows.
+// in wave order.  Every dS tile is still written by one wave.  Where it runs: on_split_rows.
 template <int D, int NP>
 constexpr int kDkdvSplitWaves = NP == 3 && D == 64 ? 2 : 4;  // what fits the 160 KB of LDS
 template <int D, int NP, bool DS = false>
@@ -1643,46 +1644,10 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_ds_kernel(DqDsArgs
 // accumulators it measured faster than two sub-blocks per wave with the fold step (bf16
 // B16 H16 T2048 d64 dQ 230.3 -> 217.9 us, B8 H16 T2048 122.9 -> 112.8; three planes at d = 32
 // within 1%, bitwise the same).
-// Whether a stage's waves should share out the streamed rows of a 32-row block, instead of each
-// walking the whole range of its own 32 rows: up to some number of 128-row workgroups, where those
-// leave CUs idle and the launch takes as long as the longest range.  Measured (us, 128-row
-// workgroups -> shared rows; Python calls, 13 us at least):
-//   bf16 d 64   B*H 4 T 1531 (48 workgroups)   dQ 26.5 -> 13.5   dK/dV 27.8 -> 18.4
-//               B*H 16 T 777 (112)                16.9 -> 14.5         18.0 -> 14.7
-//               B*H 12 T 2048 (192)               34.7 -> 24.0         36.7 -> 31.8
-//               B*H 16 T 2048 (256)               35.5 -> 29.1         37.8 -> 39.2
-//               B*H 27 T 777 (189)                17.2 -> 18.4         18.8 -> 21.8
-//   bf16 d 128  B*H 4 T 4096 (128)               113.6 -> 58.2        110.6 -> 78.3
-//               B*H 12 T 1531 (144)               48.2 -> 41.5         46.8 -> 51.4
-//               B*H 12 T 777 (84)                 27.6 -> 20.0         27.9 -> 21.8
-//               B*H 27 T 512 (108)                22.5 -> 22.5         20.5 -> 26.9
-//   bf16 d 32   B*H 12 T 4096 (384)               50.1 -> 35.5         57.9 -> 50.9
-//               B*H 48 T 1531 (576)               22.8 -> 22.9         27.9 -> 33.5
-//   x3 d 64, the whole dS-first backward: B*H 4 T 777 (28) 90 -> 69, B*H 12 T 1531 (144) 162 ->
-//   148, B*H 12 T 2048 (192) 212 -> 226, B*H 48 T 300 (144) 46 -> 45, B*H 27 T 777 (189) 94 -> 103
-//   x3 d 32, both stages: B*H 4 T 1531 (48) 130 -> 46, B*H 16 T 2048 (256) 176 -> 132, B*H 27
-//   T 1531 (324) 144 -> 157, B*H 27 T 777 (189) 75 -> 62, B*H 96 T 300 (288) 38 -> 52
-enum class Stage { Dq, Dkdv };
-bool split_rows(int D, int NP, int BH, int T, Stage stage) {
-    const bool lng = T >= 1200, dq = stage == Stage::Dq;
-    int most;
-    if (NP == 3)
-        most = D == 64 ? (lng ? 144 : T > 128 ? 112 : 64) : (lng ? 256 : T > 128 ? 176 : 48);
-    else if (T <= 256)
-        most = 0;  // the ranges are too short to share (equal times)
-    else if (D == 128)
-        most = dq ? (lng ? 192 : T >= 448 ? 112 : 48) : (lng ? 128 : T >= 600 ? 96 : 64);
-    else if (D == 64)
-        most = dq ? (lng ? 256 : 128) : (lng ? 192 : 112);
-    else
-        most = dq ? (lng ? 512 : 256) : (lng ? 320 : 256);
-    return static_cast<long long>(BH) * ((T + 127) / 128) <= most;
-}
-
 template <int D, int NP>
 void dq_dispatch(DqArgs<NP> a, hipStream_t stream) {
     if constexpr (NP == 1 || D == 32) {  // three planes at d = 64: the tiles of four waves do not fit
-        if (split_rows(D, NP, a.BH, a.T, Stage::Dq)) {
+        if (on_split_rows(Stage::Dq, NP, D, a.T, a.BH)) {
             const int n = (a.T + kSub - 1) / kSub;
             hipLaunchKernelGGL((flash_bwd_dq_split_kernel<D, NP>), dim3(a.BH * n),
                                dim3(kWave * kWaves), 0, stream, a, n);
@@ -1697,7 +1662,7 @@ void dq_dispatch(DqArgs<NP> a, hipStream_t stream) {
 
 template <int D, int NP>
 void dkdv_dispatch(DkdvArgs<NP> a, hipStream_t stream) {
-    if (split_rows(D, NP, a.BH, a.T, Stage::Dkdv)) {
+    if (on_split_rows(Stage::Dkdv, NP, D, a.T, a.BH)) {
         const int n = (a.T + kSub - 1) / kSub;
         const dim3 grid(a.BH * n), block(kWave * kDkdvSplitWaves<D, NP>);
         if constexpr (NP == 3) {

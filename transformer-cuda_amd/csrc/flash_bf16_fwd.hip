@@ -42,6 +42,7 @@
 
 #include "device_common.hpp"
 #include "bf16_tile.hpp"
+#include "forms.hpp"
 #include "launch.hpp"
 #include "sched.hpp"
 
@@ -694,7 +695,7 @@ __global__ __launch_bounds__(kWave* kWaves, D >= 128 ? 3 : 4) void flash_fwd_fol
 // 32-key tiles w, w + NW, ... of its block's range through buffers of its own (no barrier in the
 // loop), and the NW partial results meet in LDS: a quarter of the steps on four times the
 // workgroups.  A tile is copied for 32 queries instead of 128, which is why the kernels above
-// are the faster ones once they fill the chip (split_forward).  The running maximum is exact per
+// are the faster ones once they fill the chip (on_split_rows).  The running maximum is exact per
 // wave (SubState, unfolded), so m is the row's maximum.
 // ---------------------------------------------------------------------------------------
 template <int D, int NP>
@@ -864,26 +865,6 @@ void fwd_fold_launch(const FwdArgs<1>& a, hipStream_t stream) {
                        a.v, a.o, a.m_out, a.l_out, a.BH, a.T, a.scale, nblk, a.xv, a.ov, serp);
 }
 
-// Whether the waves should share out the keys: up to about a workgroup of 128 queries per two
-// CUs, per CU where the ranges are long.  Measured (us, 128-query workgroups -> shared keys;
-// Python calls, 12 us at least):
-//   bf16 d 64   B*H 12 T 1531 (144 workgroups)  21.0 -> 13.7   B*H 16 T 2048 (256)  27.3 -> 23.2
-//               B*H 12 T 4096 (384)             52.9 -> 53.4   B*H 27 T 1531 (324)  23.2 -> 28.9
-//               B*H 27 T 777 (189)              13.6 -> 13.9   B*H 1 T 4096 (32)    46.8 -> 23.2
-//   bf16 d 128  B*H 16 T 777 (112)              23.1 -> 15.8   B*H 16 T 1531 (192)  40.2 -> 34.3
-//               B*H 27 T 777 (189)              23.8 -> 29.5   B*H 16 T 2048 (256)  52.1 -> 50.9
-//   bf16 d 32   B*H 12 T 4096 (384)             39.3 -> 31.0   B*H 48 T 777 (336)   12.1 -> 12.3
-//   x3   d 64   B*H 12 T 1531 (144)             78.1 -> 58.3   B*H 16 T 2048 (256)   103 -> 95
-//               B*H 27 T 777 (189)              47.8 -> 50.2   B*H 4 T 777 (28)     41.2 -> 24.6
-//   x3   d 32   B*H 16 T 2048 (256)             68.2 -> 54.7   B*H 27 T 1531 (324)  60.4 -> 68.8
-// Up to 256 keys the ranges are too short to share (equal times).
-bool split_forward(int D, int NP, int BH, int T) {
-    if (T <= 256) return false;
-    const long long nblk = static_cast<long long>(BH) * ((T + 127) / 128);
-    if (T >= 1200) return nblk <= (NP == 1 && D == 128 ? 192 : NP == 1 && D == 32 ? 384 : 256);
-    return nblk <= (D == 32 ? 192 : NP == 3 ? 144 : 112);
-}
-
 template <int D, int NP>
 void fwd_split_launch(const FwdArgs<NP>& a, hipStream_t stream) {
     const int nblk = (a.T + kSub - 1) / kSub;
@@ -895,7 +876,7 @@ void fwd_split_launch(const FwdArgs<NP>& a, hipStream_t stream) {
 
 template <int D, int NP>
 void fwd_dispatch(const FwdArgs<NP>& a, hipStream_t stream) {
-    if (split_forward(D, NP, a.BH, a.T)) {
+    if (on_split_rows(Stage::Fwd, NP, D, a.T, a.BH)) {
         fwd_split_launch<D, NP>(a, stream);
         return;
     }

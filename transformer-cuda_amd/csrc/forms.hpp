@@ -70,4 +70,38 @@ inline bool on_shared_tiles(Stage stage, int D, int T, int BH) {
            f.step * makespan(wave, nt, wave_sum, BH, false);
 }
 
+// bf16 (planes = 1) and three planes: whether a stage's waves share out the streamed rows of one
+// 32-row block (flash_*_split_kernel) instead of each walking the whole range of its own 32 rows of
+// 128.  Sharing ends with the longest range / 4, but copies every tile for 32 rows instead of 128:
+// it is the faster form while 128-row workgroups leave CUs idle, and up to more of them the longer
+// the ranges are, as copying is then the smaller part.  So the limit on 128-row workgroups is a line
+// in T, bounded where the chip is filled either way; up to `from` keys there is too little to share
+// (equal times).  The lines lie between the last shapes that gain and the first that lose in 780
+// shapes of each type and d, from B*H 1 to 400 and T 33 to 8192, measured in both forms: none loses
+// more than 5%.  Measured (us, 128-row workgroups -> shared rows; number of workgroups):
+//   bf16 d 32   B*H 12 T 1531 (144), fwd 15.7 -> 8.8, dQ 19.0 -> 9.9, dK/dV 21.7 -> 12.4
+//               B*H 48 T 777 (336), fwd 9.7 -> 8.5, dQ 12.0 -> 10.5, dK/dV 14.3 -> 12.5
+//   bf16 d 64   B*H 12 T 1531 (144), fwd 20.2 -> 11.8, dQ 26.3 -> 15.0, dK/dV 27.7 -> 19.4
+//               B*H 27 T 777 (189), fwd 12.5 -> 11.8, dQ 16.0 -> 16.8, dK/dV 18.2 -> 20.4
+//   bf16 d 128  B*H 12 T 1024 (96), fwd 27.6 -> 15.2, dQ 33.7 -> 22.5, dK/dV 32.2 -> 27.4
+//               B*H 27 T 449 (108), fwd 15.2 -> 14.9, dQ 18.7 -> 20.7, dK/dV 19.5 -> 24.2
+//   three planes, the whole backward: d 32   B*H 16 T 2048 (256) 173 -> 127, B*H 80 T 230 (160) 31 -> 36
+//               d 64   B*H 12 T 1531 (144) 162 -> 146, B*H 24 T 1024 (192) 114 -> 126
+inline bool on_split_rows(Stage stage, int planes, int D, int T, int BH) {
+    struct Line {
+        int from, base, per, most;
+    };
+    static constexpr Line kBf16[3][3] = {  // d 32, 64, 128
+        {{256, 224, 8, 480}, {256, 190, 4, 576}, {256, 244, 15, 384}},
+        {{256, 92, 8, 320}, {256, 72, 8, 320}, {256, 60, 9, 208}},
+        {{256, 97, 16, 224}, {256, 32, 8, 192}, {256, 33, 11, 128}}};
+    static constexpr Line kThree[2][2] = {  // d 32, 64: forward, backward
+        {{288, 120, 7, 256}, {128, 94, 5, 256}}, {{256, 104, 10, 256}, {128, 108, 32, 144}}};
+    const long long nblk = static_cast<long long>(BH) * ((T - 1) / 128 + 1);
+    const int d = D == 32 ? 0 : D == 64 ? 1 : 2;
+    if (planes == 3 && stage != Stage::Fwd && T <= 128) return nblk <= (D == 32 ? 48 : 64);
+    const Line& l = planes == 3 ? kThree[d][stage != Stage::Fwd] : kBf16[d][static_cast<int>(stage)];
+    return T > l.from && nblk <= std::min(l.base + T / l.per, l.most);
+}
+
 }  // namespace tcamd

@@ -10,10 +10,11 @@
 //     (non-increasing causal work) within a head, and a group's blocks all come before the
 //     next group's.
 // And head_group at the bench shapes, with the resident capacities the occupancy query
-// reports for those kernels on MI355X; and the forms that on_shared_tiles picks at shapes where one
-// form measured clearly faster.  Prints "sched_check: all passed" on success.
+// reports for those kernels on MI355X; and the forms that on_shared_tiles and on_split_rows pick at
+// shapes where one form measured clearly faster.  Prints "sched_check: all passed" on success.
 //
-// sched_check form STAGE D T BH prints the fp32 form of a call instead (STAGE: fwd, dq, dkdv).
+// sched_check form STAGE D T BH prints the fp32 form of a call instead (STAGE: fwd, dq, dkdv),
+// sched_check form STAGE PLANES D T BH the bf16 (PLANES 1) or three-plane (3) form.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -168,20 +169,64 @@ static void check_f32_forms() {
                 for (int BH : {1, 7, 65535}) (void)tcamd::on_shared_tiles(static_cast<Stage>(st), D, T, BH);
 }
 
-static int print_form(char** a) {
+// The same for sharing rows among a workgroup's waves (three planes: the forward, and the whole
+// backward).
+static void check_split_rows() {
+    const struct {
+        Stage stage;
+        int planes, D, T, BH;
+        double block, split;
+    } measured[] = {
+        {Stage::Fwd, 1, 32, 1531, 12, 15.7, 8.8},   {Stage::Fwd, 1, 32, 1531, 48, 15.9, 17.8},
+        {Stage::Dq, 1, 32, 2048, 16, 24.4, 12.8},   {Stage::Dkdv, 1, 32, 1531, 48, 24.9, 29.2},
+        {Stage::Fwd, 1, 64, 1531, 12, 20.2, 11.8},  {Stage::Fwd, 1, 64, 1024, 24, 15.0, 12.3},
+        {Stage::Fwd, 1, 64, 777, 48, 12.8, 16.2},   {Stage::Dq, 1, 64, 1531, 12, 26.3, 15.0},
+        {Stage::Dq, 1, 64, 777, 27, 16.0, 16.8},    {Stage::Dkdv, 1, 64, 300, 36, 9.5, 10.0},
+        {Stage::Dkdv, 1, 64, 777, 12, 17.1, 13.3},  {Stage::Dkdv, 1, 64, 777, 27, 18.2, 20.4},
+        {Stage::Fwd, 1, 128, 2048, 12, 50.3, 39.3}, {Stage::Fwd, 1, 128, 777, 27, 22.5, 28.7},
+        {Stage::Dq, 1, 128, 449, 27, 18.7, 20.7},   {Stage::Dq, 1, 128, 1024, 12, 33.7, 22.5},
+        {Stage::Dkdv, 1, 128, 449, 27, 19.5, 24.2}, {Stage::Dkdv, 1, 128, 4096, 4, 108.5, 73.7},
+        {Stage::Fwd, 3, 32, 257, 64, 15.6, 17.5},   {Stage::Fwd, 3, 32, 1531, 12, 50.8, 30.7},
+        {Stage::Dkdv, 3, 32, 230, 80, 30.5, 36.4},  {Stage::Dkdv, 3, 32, 777, 27, 73.8, 60.2},
+        {Stage::Fwd, 3, 64, 230, 80, 24.6, 29.1},   {Stage::Fwd, 3, 64, 1531, 12, 75.1, 54.0},
+        {Stage::Dkdv, 3, 64, 777, 12, 90.0, 69.1},  {Stage::Dkdv, 3, 64, 1024, 24, 113.6, 126.0},
+        {Stage::Dkdv, 3, 64, 100, 40, 24.5, 21.7},
+    };
+    for (const auto& m : measured)
+        CHECK(tcamd::on_split_rows(m.stage, m.planes, m.D, m.T, m.BH) == (m.split < m.block),
+              "stage %d planes %d d %d T %d B*H %d takes the slower form (%.1f us in 128-row "
+              "workgroups, %.1f split)",
+              static_cast<int>(m.stage), m.planes, m.D, m.T, m.BH, m.block, m.split);
+    for (int st = 0; st < 3; ++st)
+        for (int planes : {1, 3})
+            for (int D : {32, 64})
+                for (int T : {1, 128, 256, 257, 8192, 2147483647})
+                    for (int BH : {1, 65535})
+                        (void)tcamd::on_split_rows(static_cast<Stage>(st), planes, D, T, BH);
+}
+
+// STAGE D T BH, or STAGE PLANES D T BH
+static int print_form(int n, char** a) {
     const char* names[] = {"fwd", "dq", "dkdv"};
     for (int st = 0; st < 3; ++st)
         if (std::strcmp(a[0], names[st]) == 0) {
-            const bool shared = tcamd::on_shared_tiles(static_cast<Stage>(st), std::atoi(a[1]),
-                                                       std::atoi(a[2]), std::atoi(a[3]));
-            std::printf("%s\n", shared ? "shared" : "per-wave");
+            const Stage stage = static_cast<Stage>(st);
+            int x[4] = {};
+            for (int i = 1; i < n; ++i) x[i - 1] = std::atoi(a[i]);
+            if (n == 4)
+                std::printf("%s\n", tcamd::on_shared_tiles(stage, x[0], x[1], x[2]) ? "shared"
+                                                                                    : "per-wave");
+            else
+                std::printf("%s\n", tcamd::on_split_rows(stage, x[0], x[1], x[2], x[3]) ? "split"
+                                                                                         : "block");
             return 0;
         }
     return 2;
 }
 
 int main(int argc, char** argv) {
-    if (argc == 6 && std::strcmp(argv[1], "form") == 0) return print_form(argv + 2);
+    if ((argc == 6 || argc == 7) && std::strcmp(argv[1], "form") == 0)
+        return print_form(argc - 2, argv + 2);
     const int bhs[] = {1, 3, 8, 12, 16, 24, 64, 96, 128, 256, 384};
     const int nbs[] = {1, 2, 7, 8, 16, 33, 64};
     for (int BH : bhs)
@@ -211,6 +256,7 @@ int main(int argc, char** argv) {
     CHECK(head_group(64, 64, 256) == 0, "BH 64: %d", head_group(64, 64, 256));
 
     check_f32_forms();
+    check_split_rows();
 
     if (failures) {
         std::printf("sched_check: %d failures\n", failures);
