@@ -1,5 +1,7 @@
 """Shared helpers of the GPU parity tests (not collected as tests)."""
 import math
+import os
+import subprocess
 
 import numpy as np
 import torch
@@ -32,3 +34,12 @@ def rel_l2(a, b):
 
 def default_scale(d):
     return 1.0 / math.sqrt(d)
+
+
+def sched(*args):
+    """The form or tile that the host's rules pick for a call (src/sched_check.cpp)."""
+    exe = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       "transformer-cuda_amd", "bin", "sched_check")
+    r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (args, r.stdout)
+    return r.stdout.strip()

@@ -75,10 +75,11 @@ def test_shapes_vs_oracle(lib, T, d):
 @pytest.mark.parametrize("B,H,T,d", [(2, 4, 300, 64), (1, 8, 160, 128), (2, 8, 383, 32),
                                      (1, 16, 640, 64), (4, 64, 200, 64)])
 def test_xcd_block_order_ragged_vs_oracle(lib, B, H, T, d):
-    """B*H a multiple of 8: every kernel maps workgroups to heads XCD by XCD (serpentine
-    rounds where the grid fits on the device at once, rank order where it does not; the
-    head groups start at config 3's size, test_config3_full), at lengths that leave the last
-    block of each head partly past T."""
+    """B*H a multiple of 8: every kernel maps workgroups to heads XCD by XCD, at lengths that leave
+    the last block of each head partly past T.  Up to 256 keys the 128-row kernels (serpentine
+    rounds: the grid fits on the device at once), beyond them the few-head kernels' plain order; the
+    128-row kernels at longer ragged T are in test_gpu_form_limits.py, the head groups start at
+    config 3's size (test_config3_full)."""
     q, k, v, do = _rounded(B, H, T, d, seed=B * H + T + d)
     scale = default_scale(d)
     want = ref.attention_fwd_bwd(q, k, v, do, scale, dtype=torch.float32)

@@ -51,8 +51,8 @@ def both_orders(lib, qkv, do, B, H, T, d, scale, merged):
     return o, two, D2, one, D1
 
 
-# (1, 2, 2048, 64) and (1, 2, 2080, 64): either side of the length where the d = 64 kernels
-# change from the shared-tile to the per-wave form
+# Few heads: the per-wave form at every length (the shared-tile form with dS, ragged and at d = 128,
+# is in test_gpu_form_limits.py)
 SHAPES = [(1, 1, 1, 64), (2, 3, 17, 32), (1, 2, 100, 64), (2, 2, 257, 128), (2, 4, 640, 64),
           (1, 1, 1000, 32), (2, 3, 300, 128), (1, 2, 2048, 64), (1, 2, 2080, 64)]
 

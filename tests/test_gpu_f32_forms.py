@@ -31,7 +31,7 @@ def attention64(q, k, v, do, scale):
     (4, 16, 1024, 64),   # 512 = two a CU, even: shared
     (4, 16, 1000, 64),   # the same, ragged
     (4, 24, 769, 64),    # 672 with a nearly empty last block: per-wave
-    (9, 16, 900, 64),    # over four a CU: shared
+    (9, 16, 900, 64),    # over four a CU: dK/dV shared, forward and dQ per-wave
     (3, 15, 1000, 128),  # 360: dK/dV shared, forward and dQ per-wave
     (8, 8, 901, 128),    # 512: all shared
     (3, 14, 700, 128),   # 252: all per-wave

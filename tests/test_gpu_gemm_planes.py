@@ -5,6 +5,8 @@ import numpy as np
 import pytest
 import torch
 
+from gpu_util import sched
+
 pytestmark = pytest.mark.gpu
 
 
@@ -21,8 +23,8 @@ def run(lib, A, B, C, M, N, K, ta, tb, alpha=1.0, beta=0.0):
     torch.cuda.synchronize()
 
 
-# (M, N, K, batch): sizes that take, in order, 256 x 256, 256 x 128, 128 x 128, 128 x 64 and
-# 64 x 64 tiles, each with ragged edges; K below, at and beyond the 16- and 32-deep chunks
+# (M, N, K, batch): 128 x 128 tiles (the first two sizes) and 64 x 64 ones, with ragged edges; K below, at and beyond the 16- and 32-deep chunks.  The
+# other tiles: test_every_tile
 @pytest.mark.parametrize("M,N,K,batch", [
     (2049, 2047, 33, 4), (1000, 1300, 47, 5), (900, 1100, 64, 4), (515, 701, 95, 4),
     (129, 65, 17, 3), (1, 1, 1, 1), (3, 130, 2, 2), (63, 64, 31, 7), (257, 2, 48, 2)])
@@ -45,6 +47,23 @@ def test_tiles_and_tails(lib, M, N, K, batch, ta, tb):
             lim = lim + 2.0 ** -22 * (beta * C.double()).abs()
         run(lib, A, B, C, M, N, K, ta, tb, alpha, beta)
         assert bool(((C.double() - exp).abs() <= lim).all()), (alpha, beta)
+
+
+@pytest.mark.parametrize("tile,M,N,K,batch", [
+    ("256x256", 1023, 1021, 1000, 16), ("256x128", 1023, 509, 1501, 12),
+    ("128x128", 1000, 1300, 47, 5), ("128x64", 1000, 500, 700, 8), ("64x64", 515, 701, 95, 4)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_every_tile(lib, tile, M, N, K, batch, ta, tb):
+    """Each tile shape with ragged rows, columns and K, at a size that the rule sends to it."""
+    assert sched("tile", M, N, batch, K, 1, 1) == f"{tile} 1"
+    g = torch.Generator(device="cuda:0").manual_seed(M + N + K)
+    A = torch.randn((batch, K, M) if ta else (batch, M, K), generator=g, device="cuda:0")
+    B = torch.randn((batch, N, K) if tb else (batch, K, N), generator=g, device="cuda:0")
+    C = torch.full((batch, M, N), float("nan"), device="cuda:0")
+    run(lib, A, B, C, M, N, K, ta, tb)
+    want, mag = product64(A, B, ta, tb)
+    # as test_tiles_and_tails
+    assert bool(((C.double() - want).abs() <= (6 * (K // 16 + 1) + 3) * 2.0 ** -23 * mag).all())
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])

@@ -3,8 +3,7 @@ loss and every parameter gradient of one forward + backward, and the clip + Adam
 for each attention mode (this build's fused path on the fp32 MFMA and on the bf16 MFMA with
 three-plane fp32 operands, the reference's tiled sequence, the reference's materialised
 default).  Shapes of config 1 (the tiny GPT), a d = 64 variant, a vocabulary of more than
-16 d_model (the split-K product of the output head's input gradient) and 4096 tokens (the
-split-K weight gradients).
+16 d_model and 4096 tokens (slices of K in the products over them).
 Tolerances are the reference's own parity gates (scripts/compare_parity.py:108-117): loss
 within 1e-5, gradients within 5e-5."""
 import numpy as np
@@ -17,10 +16,9 @@ pytestmark = pytest.mark.gpu
 
 C1 = dict(V=256, T=64, C=128, L=2, H=4, d_ff=512, B=4)
 D64 = dict(V=97, T=130, C=128, L=2, H=2, d_ff=256, B=3)
-# V >= 16 C: the output head's input gradient takes the split-K product (V = 8 * 256 + 5,
-# so the remainder product runs too)
+# a long, ragged contraction over the vocabulary: the output head's input gradient in slices of K
 VOC = dict(V=2053, T=32, C=64, L=1, H=2, d_ff=128, B=2)
-# B*T >= 4096: the weight gradients take the split-K product (four slices over the tokens)
+# 4096 tokens: the weight gradients in slices of K
 TOK = dict(V=97, T=512, C=64, L=1, H=2, d_ff=128, B=8)
 SHAPES = {"c1": C1, "d64": D64, "vocab": VOC, "tokens": TOK}
 

@@ -9,6 +9,7 @@ import torch
 
 from gpu_util import default_scale, max_abs, to_dev
 from oracle import attention_ref as ref
+from test_gpu_f32_forms import attention64
 
 pytestmark = pytest.mark.gpu
 
@@ -184,6 +185,29 @@ def test_causal_gemm_equals_full_product(lib, T, d):
             assert torch.equal(part[:, ~blk], full[:, ~blk]), f"causal {causal}"
         else:
             assert torch.equal(part, full), f"causal {causal}"
+
+
+# 13 and 14 row tiles of 64 in pairs (the middle one of 13 by itself), the last one ragged
+@pytest.mark.parametrize("T,d", [(777, 64), (833, 64), (777, 96)])
+def test_paired_row_tiles(lib, T, d):
+    """Enough heads that the triangular products take their row tiles in pairs: bitwise the full
+    product, and the whole mode against fp64."""
+    B, H = 8, 12
+    assert ((T + 63) // 64 + 1) // 2 * ((d + 63) // 64) * B * H >= 384
+    g = torch.Generator(device="cuda:0").manual_seed(T + d)
+    q, k, v, do = (torch.randn((B, H, T, d), generator=g, device="cuda:0") for _ in range(4))
+    lower = torch.tril(torch.randn((B * H, T, T), generator=g, device="cuda:0")).contiguous()
+    for ta, causal in ((False, lib.GEMM_LOWER_A), (True, lib.GEMM_UPPER_A)):
+        full, part = (torch.full((B * H, T, d), float("nan"), device="cuda:0") for _ in range(2))
+        a = (T, d, T, T * T, T * d, T * d, B * H, ta, False)
+        lib.matmul_batched_strided(lower, v, full, *a)
+        lib.matmul_batched_strided_causal(lower, v, part, *a, causal)
+        assert torch.equal(part, full)
+    scale = default_scale(d)
+    got = materialized(lib, *(x.cpu().numpy() for x in (q, k, v, do)), B, H, T, d, scale)
+    for name, exp in zip(("o", "dq", "dk", "dv"), attention64(q, k, v, do, scale)):
+        err = max_abs(got[name], exp.cpu().numpy())
+        assert err <= 1e-5, f"{name}: max-abs {err:.3e}"
 
 
 def test_materialized_equals_its_launch_sequence(lib):

@@ -1,7 +1,7 @@
 """The attention kernels whose waves share out the streamed rows of a 32-row block (few heads), in
 bf16 and for fp32 as three bf16 planes, against fp64 attention: fewer tiles than waves, one tile
-more or less than the waves' turns, ragged last tiles, and lengths either side of the rule that
-chooses them."""
+more or less than the waves' turns and ragged last tiles (bf16 up to 256 keys: the 128-row kernels).
+More heads, on either side of the rule that chooses the form: test_gpu_form_limits.py."""
 import math
 
 import pytest

@@ -14,7 +14,8 @@
 // shapes where one form measured clearly faster.  Prints "sched_check: all passed" on success.
 //
 // sched_check form STAGE D T BH prints the fp32 form of a call instead (STAGE: fwd, dq, dkdv),
-// sched_check form STAGE PLANES D T BH the bf16 (PLANES 1) or three-plane (3) form.
+// sched_check form STAGE PLANES D T BH the bf16 (PLANES 1) or three-plane (3) form, and
+// sched_check tile M N BATCH K SLICES ARRAYS the GEMM's tile and slices of K (at most SLICES).
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -22,6 +23,7 @@
 
 #include "bf16_tile.hpp"
 #include "forms.hpp"
+#include "gemm_planes.hpp"
 #include "sched.hpp"
 
 using tcamd::head_group;
@@ -224,7 +226,17 @@ static int print_form(int n, char** a) {
     return 2;
 }
 
+static int print_tile(char** a) {
+    int x[6];
+    for (int i = 0; i < 6; ++i) x[i] = std::atoi(a[i]);
+    const tcamd::gemm::Plan p = tcamd::gemm::pick_tile(x[0], x[1], x[2], x[3], x[4], x[5]);
+    const tcamd::gemm::TileRate& t = tcamd::gemm::kTiles[p.tile];
+    std::printf("%dx%d %d\n", t.bm, t.bn, p.slices);
+    return 0;
+}
+
 int main(int argc, char** argv) {
+    if (argc == 8 && std::strcmp(argv[1], "tile") == 0) return print_tile(argv + 2);
     if ((argc == 6 || argc == 7) && std::strcmp(argv[1], "form") == 0)
         return print_form(argc - 2, argv + 2);
     const int bhs[] = {1, 3, 8, 12, 16, 24, 64, 96, 128, 256, 384};
