@@ -184,7 +184,7 @@ __device__ __forceinline__ void merge_waves(f32x16 (&acc)[D / 32], f32x4* part, 
 // (the A operand ones times a statistic chunk) would cost two MFMAs per half tile.
 template <int D, int NP>
 struct DqSub {
-    bf16x8 q[D / 16][NP];  // c * Q row of query col (B operand over d)
+    bf16x8 q[D / 16][NP];  // c * Q row of query col (B operand over d); Q itself unless FOLD
     bf16x8 g[D / 16][NP];  // dO row
     f32x16 ls, ld;         // -lse2 (-1e30 for padded queries: P = 0) and -D in every row
     f32x16 acc[D / 32];    // dQ^T
@@ -221,7 +221,13 @@ __device__ __forceinline__ float chunk_dot_tree(const float* __restrict__ gp,
 // pre-multiplied by c = scale*log2 e (NP = 1: rounded to bf16, one extra rounding of ~2^-9
 // relative per element; NP = 3: in fp32, then split), so that the scores come out in the
 // log2 domain.  D = rowsum(dO o O) in fp32 from the stored O and dO.
-template <int D, int NP>
+//
+// The statistics m and l must belong to the scores that P is formed from.  The bf16 forward takes
+// them from c*Q rounded as here, but for few heads (flash_fwd_split_kernel) from the products of Q
+// itself: then (FOLD = false) Q stays as it is, and c is applied to the sums.  With rounded scores
+// against those statistics dQ's error was 3.1e-3 of its norm instead of 2.9e-3, 8.9e-3 instead of
+// 6.0e-3 with scores of 4 times the variance (d 64, T 1531).
+template <int D, int NP, bool FOLD = true>
 __device__ __forceinline__ void dq_init(DqSub<D, NP>& sb, const InT<NP>* __restrict__ qh,
                                         const InT<NP>* __restrict__ oh,
                                         const InT<NP>* __restrict__ gh,
@@ -244,7 +250,7 @@ __device__ __forceinline__ void dq_init(DqSub<D, NP>& sb, const InT<NP>* __restr
         part = chunk_dot_tree<D>(gh + static_cast<size_t>(qi) * ors,
                                  oh + static_cast<size_t>(qi) * ors, half);
     }
-    load_operand<D, NP, true>(sb.q, qh, qi, T, half, qrs, c);
+    load_operand<D, NP, FOLD>(sb.q, qh, qi, T, half, qrs, c);
     const float dlt = xhalf_sum(part);
     float nl = -1e30f;
     if (qi < T) {
@@ -282,20 +288,26 @@ __device__ __forceinline__ void dq_ds(f32x16& s, const f32x16& dp, bf16x8 (&db)[
 
 // One 32-key half tile of the wave's sub-block (MASK: its diagonal one).  ka/va: this lane's
 // row-read addresses in plane 0 of the K / V tile; kta: transposing-read addresses in plane
-// 0 of the K tile; plane i lies i tile sizes further.  S^T and dP^T start from -lse2 and -D.
-template <int D, int NP, bool MASK>
+// 0 of the K tile; plane i lies i tile sizes further.  S^T and dP^T start from -lse2 and -D (FOLD),
+// or S^T from 0, to become c S^T - lse2.
+template <int D, int NP, bool MASK, bool FOLD = true>
 __device__ __forceinline__ void dq_half(int kb, const uint32_t (&ka)[D / 16],
                                         const uint32_t (&va)[D / 16],
                                         const uint32_t (&kta)[D / 32], DqSub<D, NP>& sb, int qj,
-                                        int col, int half) {
+                                        int col, int half, float c) {
     constexpr uint32_t kPlane = Swz<D, kKeyTileDq<NP>>::kBytes;
-    f32x16 s = sb.ls;
+    f32x16 s = f32x16{};
+    if constexpr (FOLD) s = sb.ls;
 #pragma unroll
     for (int st = 0; st < D / 16; ++st) {
         bf16x8 a[NP];
 #pragma unroll
         for (int i = 0; i < NP; ++i) a[i] = lds_b128(ka[st] + i * kPlane);
         s = mma_planes<NP>(a, sb.q[st], s);
+    }
+    if constexpr (!FOLD) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = fmaf(s[r], c, sb.ls[0]);
     }
     f32x16 p = sb.ld;
 #pragma unroll
@@ -339,7 +351,7 @@ struct DqArgs {
 };
 
 // 128 queries per workgroup, wave w owns the 32-query sub-block w.
-template <int D, int NP>
+template <int D, int NP, bool FOLD>
 __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_bf16_kernel(DqArgs<NP> a,
                                                                          int nblk) {
     constexpr int KT = kKeyTileDq<NP>;
@@ -383,7 +395,7 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_bf16_kernel(DqArgs
     copy_tile(0);
 
     DqSub<D, NP> sb;
-    dq_init<D, NP>(sb, a.q + qoff, a.o + ooff, a.dO + ooff, a.m, a.l, a.Dws, a.qv.row,
+    dq_init<D, NP, FOLD>(sb, a.q + qoff, a.o + ooff, a.dO + ooff, a.m, a.l, a.Dws, a.qv.row,
                    a.ov.row, stat_off, qj + col, T, half, c);
     if constexpr (NP > 1) {
         if (a.gp != nullptr) store_planes<D, NP>(a.gp + koff, a.pstride, sb.g, qj + col, T, half);
@@ -417,11 +429,11 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_bf16_kernel(DqArgs
     int hh = 0;
     for (; hh + 1 < hB; ++hh) {
         tile_sync(hh);
-        dq_half<D, NP, false>(32 * hh, ka, va, kta, sb, qj, col, half);
+        dq_half<D, NP, false, FOLD>(32 * hh, ka, va, kta, sb, qj, col, half, c);
     }
     if (hh < hB) {
         tile_sync(hh);
-        dq_half<D, NP, true>(32 * hh, ka, va, kta, sb, qj, col, half);
+        dq_half<D, NP, true, FOLD>(32 * hh, ka, va, kta, sb, qj, col, half, c);
         ++hh;
     }
     for (; hh < hend; ++hh) tile_sync(hh);
@@ -439,7 +451,7 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_bf16_kernel(DqArgs
 // Stage 1 for few heads: the waves of a workgroup share out the keys of one 32-query block
 // through K and V tiles of their own, and their partial dQ meet in LDS, in wave order (as the
 // forward's flash_fwd_split_kernel; where it runs: on_split_rows).
-template <int D, int NP>
+template <int D, int NP, bool FOLD>
 __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_split_kernel(DqArgs<NP> a, int nblk) {
     using S = Swz<D, 32>;
     constexpr int NW = kWaves;
@@ -477,7 +489,7 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_split_kernel(DqArg
     if (wave < ntile) copy_tile(wave, 0);
     // every wave forms D and the statistics of its 32 queries (and stores the same D)
     DqSub<D, NP> sb;
-    dq_init<D, NP>(sb, a.q + a.qv.off(bh), a.o + ooff, a.dO + ooff, a.m, a.l, a.Dws, a.qv.row,
+    dq_init<D, NP, FOLD>(sb, a.q + a.qv.off(bh), a.o + ooff, a.dO + ooff, a.m, a.l, a.Dws, a.qv.row,
                    a.ov.row, static_cast<size_t>(bh) * T, qj + col, T, half, c);
     uint32_t roff[D / 16], troff[D / 32];
     lane_offsets<D>(lane, roff, troff);
@@ -501,9 +513,9 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_split_kernel(DqArg
 #pragma unroll
         for (int i = 0; i < D / 32; ++i) kta[i] = at + troff[i];
         if (kt + 1 < ntile)
-            dq_half<D, NP, false>(32 * kt, ka, va, kta, sb, qj, col, half);
+            dq_half<D, NP, false, FOLD>(32 * kt, ka, va, kta, sb, qj, col, half, c);
         else
-            dq_half<D, NP, true>(32 * kt, ka, va, kta, sb, qj, col, half);
+            dq_half<D, NP, true, FOLD>(32 * kt, ka, va, kta, sb, qj, col, half, c);
     }
     __syncthreads();  // no wave reads its tiles any more
     merge_waves<D, NW>(sb.acc, reinterpret_cast<f32x4*>(&sm[0]), wave, lane);
@@ -1644,20 +1656,31 @@ __global__ __launch_bounds__(kWave* kWaves) void flash_bwd_dq_ds_kernel(DqDsArgs
 // accumulators it measured faster than two sub-blocks per wave with the fold step (bf16
 // B16 H16 T2048 d64 dQ 230.3 -> 217.9 us, B8 H16 T2048 122.9 -> 112.8; three planes at d = 32
 // within 1%, bitwise the same).
-template <int D, int NP>
-void dq_dispatch(DqArgs<NP> a, hipStream_t stream) {
+template <int D, int NP, bool FOLD>
+void dq_launch(DqArgs<NP> a, hipStream_t stream) {
     if constexpr (NP == 1 || D == 32) {  // three planes at d = 64: the tiles of four waves do not fit
         if (on_split_rows(Stage::Dq, NP, D, a.T, a.BH)) {
             const int n = (a.T + kSub - 1) / kSub;
-            hipLaunchKernelGGL((flash_bwd_dq_split_kernel<D, NP>), dim3(a.BH * n),
+            hipLaunchKernelGGL((flash_bwd_dq_split_kernel<D, NP, FOLD>), dim3(a.BH * n),
                                dim3(kWave * kWaves), 0, stream, a, n);
             return;
         }
     }
     const int nblk = (a.T + kWaves * kSub - 1) / (kWaves * kSub);
-    const auto kernel = flash_bwd_dq_bf16_kernel<D, NP>;
+    const auto kernel = flash_bwd_dq_bf16_kernel<D, NP, FOLD>;
     a.serp = a.BH * nblk <= resident_capacity(kernel, kWave * kWaves, 0) ? 1 : 0;
     hipLaunchKernelGGL(kernel, dim3(a.BH * nblk), dim3(kWave * kWaves), 0, stream, a, nblk);
+}
+
+template <int D, int NP>
+void dq_dispatch(const DqArgs<NP>& a, hipStream_t stream) {
+    if constexpr (NP == 1) {
+        if (on_split_rows(Stage::Fwd, NP, D, a.T, a.BH)) {  // whose statistics are not folded
+            dq_launch<D, NP, false>(a, stream);
+            return;
+        }
+    }
+    dq_launch<D, NP, true>(a, stream);
 }
 
 template <int D, int NP>
