@@ -13,7 +13,9 @@
  *     and left at zero when the launch ends; so at most 64 launches of one family may run
  *     at the same time (on different streams).  A launch captured into a graph takes no
  *     slot (it runs a static schedule), so replays of a graph, concurrent or not, share
- *     nothing.  The results do not depend on the schedule (bitwise);
+ *     nothing.  The results do not depend on the schedule (bitwise).  They may depend on B*H: the
+ *     forward and backward stages come in two forms each, chosen by B*H, T and d_head, which round
+ *     differently, so that a sequence need not give the same bits in batches of different sizes;
  *   - attn_tiled_causal_backward_f32_noalloc keeps D in a scratch array shared by every
  *     call on the same GPU (see there).
  *
@@ -138,7 +140,12 @@ int attn_causal_softmax_backward_blocked_f32(const float* dprobs, const float* p
  *   C[b*strideC] (M x N, ldc = N) = alpha * op(A[b*strideA]) * op(B[b*strideB]) + beta * C
  * op(A) = A (M x K, lda = K) or, if transA, A^T of A stored K x M (lda = M); op(B) = B (K x N,
  * ldb = N) or, if transB, B^T of B stored N x K (ldb = K).  beta == 0 does not read C.
- * Strides >= 0; alpha, beta finite (else ATTN_ERROR_INVALID_VALUE).  No alignment needed. */
+ * Strides >= 0; alpha, beta finite (else ATTN_ERROR_INVALID_VALUE).  No alignment needed.
+ * Precision: fp32's over its whole range, subnormal numbers included.  A product of two elements is
+ * taken as six of its nine plane products, the rest being below 2^-26 of it, and sums are rounded
+ * to fp32 once for every 16 products and plane product, more accurate from K = 4 on than a chain of
+ * fp32 roundings; up to K = 3 it is the fp32 MFMA's.  Outputs that infinities, elements from 2^104
+ * or sums from 2^80 touch are taken on the fp32 MFMA, in blocks of 32 x 32, at its lower rate. */
 int attn_matmul_batched_strided_f32(const float* A, const float* B, float* C, int M, int N,
                                     int K, long long strideA, long long strideB,
                                     long long strideC, int batch_count, int transA, int transB,

@@ -5,7 +5,8 @@
  * projection, causal attention, out projection + residual, LayerNorm, FFN with tanh GELU +
  * residual), final LayerNorm, LM head, mean cross-entropy, and the fused clip + AdamW +
  * zero-grad optimizer step (src/optimizer.cu:117-154, driven as in src/benchmark.cu:195).
- * fp32 throughout; GEMMs on the bf16 MFMA, fp32 operands as three bf16 planes; the attention through libtcamd_attn (attn_capi.h).
+ * fp32 throughout; GEMMs on the bf16 MFMA, fp32 operands as three bf16 planes (precision as
+ * attn_matmul_batched_strided_f32's); the attention through libtcamd_attn (attn_capi.h).
  *
  * Parameters live in one flat buffer in the reference's order (src/model.cu:185-217):
  * tok_emb (V,C), pos_emb (T,C), per layer [ln1 gamma, beta (C), qkv_w (C,3C), qkv_b (3C),

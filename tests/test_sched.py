@@ -1,8 +1,9 @@
-"""The kernels' workgroup -> (head, block) orders and the host's head-group rule, checked on
-the CPU by transformer-cuda_amd/bin/sched_check (built from src/sched_check.cpp with the
+"""The kernels' workgroup -> (head, block) orders and the host's rules for head groups and for the
+forms of the attention stages, checked on the CPU by transformer-cuda_amd/bin/sched_check (built from src/sched_check.cpp with the
 kernels' own headers): every order is a bijection onto the (head, block) pairs, keeps a
-head's blocks on one XCD when the head count allows, takes blocks heaviest first, and
-head_group picks the groups measured at the bench shapes."""
+head's blocks on one XCD when the head count allows, takes blocks heaviest first,
+head_group picks the groups measured at the bench shapes, and the forms are the ones that measured
+clearly faster."""
 import os
 import subprocess
 
