@@ -142,7 +142,7 @@ int attn_causal_softmax_backward_blocked_f32(const float* dprobs, const float* p
  * ldb = N) or, if transB, B^T of B stored N x K (ldb = K).  beta == 0 does not read C.
  * Strides >= 0; alpha, beta finite (else ATTN_ERROR_INVALID_VALUE).  No alignment needed.
  * Precision: fp32's over its whole range, subnormal numbers included.  A product of two elements is
- * taken as six of its nine plane products, the rest being below 2^-26 of it, and sums are rounded
+ * taken as six of its nine plane products, the rest being below 2^-23 of it, and sums are rounded
  * to fp32 once for every 16 products and plane product, more accurate from K = 4 on than a chain of
  * fp32 roundings; up to K = 3 it is the fp32 MFMA's.  Outputs that infinities, elements from 2^104
  * or sums from 2^80 touch are taken on the fp32 MFMA, in blocks of 32 x 32, at its lower rate. */
